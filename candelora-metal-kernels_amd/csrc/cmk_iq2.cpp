@@ -175,8 +175,8 @@ size_t workspace_for(Path p, int variant, bool w8a8, int x_dtype, size_t m, uint
   if (base > 0 && cmk::iq_mm_rows_per_pass(x_dtype, w8a8, nullptr, (uint32_t)m, out_dim, in_dim,
                                            any, base) == m)
     return base;
-  return std::max(base, cmk::iq_mm_scratch_bytes(x_dtype, w8a8, nullptr, (uint32_t)m, out_dim,
-                                                 in_dim));
+  return std::max(base, cmk::iq_mm_scratch_bytes(x_dtype, w8a8, p == Path::Gemm, nullptr,
+                                                 (uint32_t)m, out_dim, in_dim));
 }
 
 // Shared validation of cmk_iq2_matmul / cmk_iq2_matmul_workspace_size.

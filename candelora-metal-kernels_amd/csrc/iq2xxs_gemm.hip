@@ -548,10 +548,10 @@ size_t gemm_f32_scratch_bytes(uint32_t m, uint32_t in_dim, bool w8a8) {
   return (w8a8 ? 1 : 2) * (size_t)m * in_dim * 2;
 }
 
-// Sum of the k-split partials in split order (deterministic).  The loads of
-// up to kReduceBatch splits are issued before their adds, so a thread waits
-// for one memory round trip per batch rather than one per split; the adds
-// keep split order.
+// Sum of the k-split partials in split order (deterministic), in 64 bits and rounded
+// once: 16 partials added in fp32 lose 7.6e-8 of the result, as much as the partials
+// themselves.  The loads of up to kReduceBatch splits are issued before their adds, so
+// a thread waits for one memory round trip per batch rather than one per split.
 constexpr uint32_t kReduceBatch = 16;
 
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __restrict__ part,
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __r
                                                                 const float* __restrict__ gate) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x) {
-    float v = part[i];
+    double sum = part[i];
     for (uint32_t zb = 1; zb < splits; zb += kReduceBatch) {
       float w[kReduceBatch];
 #pragma unroll
@@ -568,8 +568,9 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __r
         if (zb + j < splits) w[j] = part[(uint64_t)(zb + j) * n + i];
 #pragma unroll
       for (uint32_t j = 0; j < kReduceBatch; ++j)
-        if (zb + j < splits) v += w[j];
+        if (zb + j < splits) sum += w[j];
     }
+    const float v = (float)sum;
     out[i] = gate ? silu_mul(gate[i], v) : v;
   }
 }
@@ -581,7 +582,8 @@ __global__ __launch_bounds__(256) void gemm_split_reduce4_kernel(const float4* _
                                                                  const float4* __restrict__ gate) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4;
        i += (uint64_t)gridDim.x * blockDim.x) {
-    float4 v = part[i];
+    const float4 first = part[i];
+    double sx = first.x, sy = first.y, sz = first.z, sw = first.w;
     for (uint32_t zb = 1; zb < splits; zb += kReduceBatch) {
       float4 w[kReduceBatch];
 #pragma unroll
@@ -590,13 +592,14 @@ __global__ __launch_bounds__(256) void gemm_split_reduce4_kernel(const float4* _
 #pragma unroll
       for (uint32_t j = 0; j < kReduceBatch; ++j) {
         if (zb + j < splits) {
-          v.x += w[j].x;
-          v.y += w[j].y;
-          v.z += w[j].z;
-          v.w += w[j].w;
+          sx += w[j].x;
+          sy += w[j].y;
+          sz += w[j].z;
+          sw += w[j].w;
         }
       }
     }
+    float4 v = make_float4((float)sx, (float)sy, (float)sz, (float)sw);
     if (gate) {
       const float4 g = gate[i];
       v = make_float4(silu_mul(g.x, v.x), silu_mul(g.y, v.y), silu_mul(g.z, v.z),

@@ -114,8 +114,8 @@ bool iq_mm_pays(int variant, int x_dtype, bool w8a8, size_t m, uint32_t out_dim,
                 uint32_t in_dim);
 bool iq_mm_supported(int variant, const uint8_t* wb, const uint8_t* ws, uint32_t out_dim,
                      uint32_t in_dim);
-size_t iq_mm_scratch_bytes(int x_dtype, bool w8a8, const void* x, uint32_t m, uint32_t out_dim,
-                           uint32_t in_dim);
+size_t iq_mm_scratch_bytes(int x_dtype, bool w8a8, bool f16_weights, const void* x, uint32_t m,
+                           uint32_t out_dim, uint32_t in_dim);
 uint32_t iq_mm_rows_per_pass(int x_dtype, bool w8a8, const void* x, uint32_t m, uint32_t out_dim,
                              uint32_t in_dim, const void* scratch, size_t budget);
 hipError_t launch_iq_mm(int variant, bool f16_weights, const void* x, int x_dtype, bool w8a8,
