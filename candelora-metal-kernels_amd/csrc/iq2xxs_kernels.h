@@ -109,13 +109,17 @@ hipError_t launch_iq_stage_rows(const void* x, int x_dtype, bool w8a8, uint32_t 
 // in passes of iq_mm_rows_per_pass; 0 where neither 128 rows nor the fewer there are fit.
 // f16_weights (variant 0): weights rounded once to f16, as the GEMM has them.  gate
 // non-null: out = silu(gate) * (x . w).
-// iq_mm_pays: the shapes where it is the faster kernel.
+// iq_mm_pays: the shapes where it is the faster kernel.  iq_mm_scratch_serves: whether
+// `budget` bytes hold all rows, and enough of the split to take no more than a third longer
+// than at best.
 bool iq_mm_pays(int variant, int x_dtype, bool w8a8, size_t m, uint32_t out_dim,
                 uint32_t in_dim);
 bool iq_mm_supported(int variant, const uint8_t* wb, const uint8_t* ws, uint32_t out_dim,
                      uint32_t in_dim);
 size_t iq_mm_scratch_bytes(int x_dtype, bool w8a8, bool f16_weights, const void* x, uint32_t m,
                            uint32_t out_dim, uint32_t in_dim);
+bool iq_mm_scratch_serves(int x_dtype, bool w8a8, bool f16_weights, uint32_t m, uint32_t out_dim,
+                          uint32_t in_dim, size_t budget);
 uint32_t iq_mm_rows_per_pass(int x_dtype, bool w8a8, const void* x, uint32_t m, uint32_t out_dim,
                              uint32_t in_dim, const void* scratch, size_t budget);
 hipError_t launch_iq_mm(int variant, bool f16_weights, const void* x, int x_dtype, bool w8a8,

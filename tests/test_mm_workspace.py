@@ -1,0 +1,14 @@
+"""The workspace query for calls that the register-dequantising matmul takes (host only)."""
+
+
+def test_query_has_room_for_the_split(cabi):
+    """Few rows of a long K: staged rows and the partial sums of K split in four, where the
+    decode launches' own split would hold the rows but not the partials."""
+    for v, x, m, staged in ((cabi.CMK_IQ2_XS, cabi.CMK_BF16, 8, True),
+                            (cabi.CMK_IQ2_S, cabi.CMK_BF16, 5, True),
+                            (cabi.CMK_IQ3_S, cabi.CMK_BF16, 12, True),
+                            (cabi.CMK_IQ2_XS, cabi.CMK_F16, 2, False),
+                            (cabi.CMK_IQ2_XXS, cabi.CMK_BF16, 16, True)):
+        rows = 256 + m * 14336 * 2 if staged else 0
+        rows = (rows + 255) // 256 * 256
+        assert cabi.workspace_size(x, m, 4096, 14336, variant=v) == rows + 4 * m * 4096 * 4
