@@ -163,10 +163,13 @@ template <int XD, int kMode>
 static hipError_t launch_stage(const void* x, uint32_t m, uint32_t in_dim, uint32_t pitch,
                                float* row_inv, uint16_t* q, hipStream_t stream) {
   // An octet a thread for few rows (the round trip counts); for many, workgroups of 256,
-  // several to a CU (2048 rows of 4096, bf16: 10.3 us).
+  // several to a CU (2048 rows of 4096, bf16: 10.3 us), where they hold the row: past 16384
+  // columns they would read it twice (IQ2_XXS matmuls of 2048 x 512 x 28672, staging
+  // included, rows read twice / held: f32 289 / 250 us, bf16 139 / 124, f32 W8A8 192 / 147).
   const uint32_t octets = pitch / 8;
-  const uint32_t threads =
-      m > 512 ? 256 : std::min(kStageThreads, std::max(256u, (octets + 63) / 64 * 64));
+  const uint32_t threads = m > 512 && octets <= 256 * 8
+                               ? 256
+                               : std::min(kStageThreads, std::max(256u, (octets + 63) / 64 * 64));
   const uint32_t per = (octets + threads - 1) / threads;
   auto kern = per <= 1   ? &iq_stage_rows_kernel<XD, kMode, 1>
               : per <= 2 ? &iq_stage_rows_kernel<XD, kMode, 2>
