@@ -12,3 +12,10 @@ def test_query_has_room_for_the_split(cabi):
         rows = 256 + m * 14336 * 2 if staged else 0
         rows = (rows + 255) // 256 * 256
         assert cabi.workspace_size(x, m, 4096, 14336, variant=v) == rows + 4 * m * 4096 * 4
+
+
+def test_query_counts_row_pairs_past_2_31(cabi):
+    """f32 rows are staged as pairs, 2^32 and more of them from 2^31 rows on."""
+    def query(m):
+        return cabi.workspace_size(cabi.CMK_F32, m, 2, 8, variant=cabi.CMK_IQ2_XS)
+    assert query((1 << 31) + 64) >= query((1 << 31) - 64)
