@@ -169,7 +169,9 @@ size_t workspace_for(Path p, int variant, bool w8a8, int x_dtype, size_t m, uint
   const size_t req = workspace_required(p, w8a8, x_dtype, m, out_dim, in_dim);
   const size_t split = rows_split_bytes(p, w8a8, m, out_dim, in_dim, kMaxCusForQuery);
   const size_t base = split ? split_offset(req) + split : req;
-  if (!mm_shape(variant, w8a8, x_dtype, m, out_dim, in_dim)) return base;
+  if (!mm_shape(variant, w8a8, x_dtype, m, out_dim, in_dim) ||
+      !cmk::iq_mm_supported(variant, nullptr, nullptr, out_dim, in_dim))
+    return base;
   // (decode-shaped IQ2_XXS of few weights gains nothing from a split)
   if (variant == CMK_IQ2_XXS && m <= kGemvMaxM && (uint64_t)out_dim * in_dim <= 1u << 22)
     return base;

@@ -105,8 +105,9 @@ hipError_t launch_iq_stage_rows(const void* x, int x_dtype, bool w8a8, uint32_t 
 // MFMA matmul with exact weights, dequantised in registers (variant 0 .. 3, any m).
 // Needs weight_bytes 16-byte and weight_scales 2-byte aligned and below 2 GB
 // (iq_mm_supported), and scratch (16-byte aligned) for staged rows and k-split partials:
-// at best iq_mm_scratch_bytes.  With less (`budget` bytes) K is split less, and the rows go
-// in passes of iq_mm_rows_per_pass; 0 where neither 128 rows nor the fewer there are fit.
+// at best iq_mm_scratch_bytes (of one pass: staged rows go in passes of 256 MB; 0 where none
+// would serve).  With less (`budget` bytes) K is split less, and the rows go in passes of
+// iq_mm_rows_per_pass; 0 where neither 128 rows nor the fewer there are fit.
 // f16_weights (variant 0): weights rounded once to f16, as the GEMM has them.  gate
 // non-null: out = silu(gate) * (x . w).
 // iq_mm_pays: the shapes where it is the faster kernel.  iq_mm_scratch_serves: whether

@@ -19,3 +19,17 @@ def test_query_counts_row_pairs_past_2_31(cabi):
     def query(m):
         return cabi.workspace_size(cabi.CMK_F32, m, 2, 8, variant=cabi.CMK_IQ2_XS)
     assert query((1 << 31) + 64) >= query((1 << 31) - 64)
+
+
+def test_query_is_bounded(cabi):
+    """Staged rows of one pass (256 MB and their scales), not of all rows; and nothing more
+    than the decode launches' split where the matmul cannot run: rows too long for its 32-bit
+    offsets, 2 GB of weights and more."""
+    mb = 1 << 20
+    for x in (cabi.CMK_F32, cabi.CMK_BF16):
+        rows = 256 * mb // (28672 * (4 if x == cabi.CMK_F32 else 2)) // 128 * 128
+        bytes_ = rows * 28672 * (4 if x == cabi.CMK_F32 else 2)
+        got = cabi.workspace_size(x, 65536, 28672, 28672, variant=cabi.CMK_IQ2_XS)
+        assert bytes_ < got <= 256 * mb + 4 * rows + 256
+    assert cabi.workspace_size(cabi.CMK_F32, 200, 1, 8 * mb, variant=cabi.CMK_IQ2_XS) <= 4 * mb
+    assert cabi.workspace_size(cabi.CMK_F32, 200, 1 << 18, 32768, variant=cabi.CMK_IQ2_XS) <= 4 * mb
