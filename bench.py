@@ -538,7 +538,7 @@ def bench_configs(pkg, torch, stream):
                 c()
             us = _timed_graph(torch, cabi, stream, sh, lambda i: calls[i % copies](), 100)
             gbs = alg_bytes(m, k, n) / (us * 1e-6) / 1e9
-            path = cabi.matmul_path(cabi.CMK_F32, m, n, k, cabi.CMK_ACT_QUANT_W8A8)
+            path = cabi.matmul_kernel(cabi.CMK_F32, m, n, k, mode=cabi.CMK_ACT_QUANT_W8A8)["kernel"]
             res["config2_w8a8"].append({"m": m, "k": k, "n": n, "us": us, "gbs": gbs,
                                         "path": path, "frac_of_hbm_peak": gbs / HBM_PEAK_GBS})
             log(f"[bench] config 2 W8A8 m={m} k={k} n={n} ({path}): {us:.2f} us, "
@@ -831,7 +831,7 @@ def main():
 
     if args.gpus != 1:
         print(f"bench.py: --gpus {args.gpus} requested, but this build measures one GPU only "
-              "(the IQ2_XXS path is single-GPU; see DESIGN.md for how it would shard).",
+              "(the IQ2_XXS path is single-GPU).",
               file=sys.stderr)
         sys.exit(2)
 
@@ -929,7 +929,7 @@ def main():
         line["mlp_step_m1"] = mlp
     if configs is not None:
         line["config2_small_m"] = configs["config2"]
-        line["config2_w8a8_int8"] = configs["config2_w8a8"]
+        line["config2_w8a8"] = configs["config2_w8a8"]
         line["config4_70b_layer"] = configs["config4"]
     if not args.no_cpu_baseline:
         line["cpu_baseline"] = cpu_baseline(pkg, args.cpu_seconds)

@@ -36,6 +36,7 @@ EXPORTED = (
     "cmk_last_error",
     "cmk_abi_version",
     "cmk_iq2_matmul_path",
+    "cmk_iq2_matmul_kernel",
     "cmk_device_count",
     "cmk_set_device",
     "cmk_device_props",
@@ -95,6 +96,9 @@ def lib() -> ctypes.CDLL:
     L.cmk_abi_version.restype = I
     L.cmk_iq2_matmul_path.argtypes = [I, S, S, S, I]
     L.cmk_iq2_matmul_path.restype = I
+    L.cmk_iq2_matmul_kernel.argtypes = [I, S, S, S, I, I, S, ctypes.POINTER(S), ctypes.POINTER(I),
+                                        ctypes.POINTER(I)]
+    L.cmk_iq2_matmul_kernel.restype = I
     L.cmk_device_count.argtypes = [ctypes.POINTER(I)]
     L.cmk_set_device.argtypes = [I]
     L.cmk_device_props.argtypes = [ctypes.c_char_p, S, ctypes.POINTER(I), ctypes.POINTER(S),
@@ -178,7 +182,24 @@ def dequantize_raw(wb_ptr, wb_len, ws_ptr, ws_len, out_dim, in_dim, out_ptr,
 
 
 def matmul_path(x_dtype, m, out_dim, in_dim, mode=CMK_ACT_QUANT_OFF) -> str:
+    """IQ2_XXS: "gemv" where the weights are exact, "gemm" where they are rounded to f16."""
     return "gemm" if lib().cmk_iq2_matmul_path(x_dtype, m, out_dim, in_dim, mode) == 1 else "gemv"
+
+
+def matmul_kernel(x_dtype, m, out_dim, in_dim, variant=CMK_IQ2_XXS, mode=CMK_ACT_QUANT_OFF,
+                  workspace_bytes=None) -> dict:
+    """The kernel that serves aligned buffers with this workspace (None: as much as it can
+    use): "decode", "gemm" or "register_matmul", the last with its rows per pass, row tile
+    and splits of K."""
+    rows, tile, splits = ctypes.c_size_t(0), ctypes.c_int(0), ctypes.c_int(0)
+    rc = lib().cmk_iq2_matmul_kernel(
+        x_dtype, m, out_dim, in_dim, variant, mode,
+        ctypes.c_size_t(-1).value if workspace_bytes is None else workspace_bytes,
+        ctypes.byref(rows), ctypes.byref(tile), ctypes.byref(splits))
+    if rc < 0:
+        check(rc)
+    return {"kernel": ("decode", "gemm", "register_matmul")[rc], "rows_per_pass": rows.value,
+            "row_tile": tile.value, "splits": splits.value}
 
 
 def device_props() -> dict:

@@ -337,6 +337,45 @@ int cmk_iq2_matmul_path(cmk_dtype x_dtype, size_t m, size_t out_dim, size_t in_d
              : 0;
 }
 
+int cmk_iq2_matmul_kernel(cmk_dtype x_dtype, size_t m, size_t out_dim, size_t in_dim,
+                          cmk_iq2_variant variant, cmk_act_quant_mode mode,
+                          size_t workspace_bytes, size_t* rows_per_pass, int* row_tile,
+                          int* splits) {
+  int md = (int)mode;
+  Dims dims;
+  const int rc = validate_matmul((int)x_dtype, m, out_dim, in_dim, (int)variant, &md, 0, 0, 0,
+                                 false, &dims);
+  if (rc != CMK_OK) return rc;
+  const bool w8a8 = md == CMK_ACT_QUANT_W8A8;
+  const Path p = variant != CMK_IQ2_XXS
+                     ? Path::Variant
+                     : choose_path((int)x_dtype, m, dims.out_dim, dims.in_dim, nullptr, nullptr,
+                                   nullptr, w8a8);
+  const size_t need = workspace_required(p, w8a8, (int)x_dtype, m, dims.out_dim, dims.in_dim);
+  if (m > 0 && workspace_bytes < need)
+    return fail(CMK_ERR_INVALID_ARGUMENT,
+                "iq2_matmul workspace too small: got %zu expected at least %zu (see "
+                "cmk_iq2_matmul_workspace_size)",
+                workspace_bytes, need);
+  const bool one_row =
+      p == Path::Variant && m == 1 &&
+      cmk::iq_variant_gemv_fits((int)variant, nullptr, nullptr, nullptr, dims.out_dim, dims.in_dim,
+                                (int)x_dtype, kMaxCusForQuery);
+  MmUse mm = {0, 0};
+  if (m > 0 && !one_row)
+    mm = mm_use(p, (int)variant, nullptr, (int)x_dtype, w8a8, nullptr, nullptr, dims,
+                reinterpret_cast<const void*>(kWorkspaceAlign), workspace_bytes);
+  int tile = 0, parts = 0;
+  if (mm.rows > 0)
+    cmk::iq_mm_shape((int)x_dtype, w8a8, p == Path::Gemm, std::min(dims.m, mm.rows), dims.out_dim,
+                     dims.in_dim, mm.budget, &tile, &parts);
+  if (rows_per_pass) *rows_per_pass = mm.rows;
+  if (row_tile) *row_tile = tile;
+  if (splits) *splits = parts;
+  (void)ok();
+  return mm.rows > 0 ? 2 : p == Path::Gemm ? 1 : 0;
+}
+
 int cmk_iq2_matmul(const void* x, cmk_dtype x_dtype, size_t x_len, size_t m,
                    const uint8_t* weight_bytes, size_t weight_bytes_len,
                    const uint8_t* weight_scales, size_t weight_scales_len, size_t out_dim,

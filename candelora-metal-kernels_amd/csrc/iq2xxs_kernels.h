@@ -123,6 +123,9 @@ bool iq_mm_scratch_serves(int x_dtype, bool w8a8, bool f16_weights, uint32_t m, 
                           uint32_t in_dim, size_t budget);
 uint32_t iq_mm_rows_per_pass(int x_dtype, bool w8a8, const void* x, uint32_t m, uint32_t out_dim,
                              uint32_t in_dim, const void* scratch, size_t budget);
+// Tile rows (staged rows for f32 without W8A8) and k splits of a pass of `rows` aligned rows.
+void iq_mm_shape(int x_dtype, bool w8a8, bool f16_weights, uint32_t rows, uint32_t out_dim,
+                 uint32_t in_dim, size_t budget, int* row_tile, int* splits);
 hipError_t launch_iq_mm(int variant, bool f16_weights, const void* x, int x_dtype, bool w8a8,
                         uint32_t m, const uint8_t* wb, const uint8_t* ws, float* out, uint32_t out_dim,
                         uint32_t in_dim, uint32_t rows_per_pass, void* scratch, size_t budget,

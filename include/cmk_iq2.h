@@ -235,10 +235,23 @@ int cmk_iq2_matmul_swiglu(const void *x, cmk_dtype x_dtype, size_t x_len, size_t
 const char *cmk_last_error(void);
 /* CMK_IQ2_ABI_VERSION of the loaded library. */
 int cmk_abi_version(void);
-/* Which kernel family cmk_iq2_matmul picks for these arguments:
- * 0 = GEMV (small m), 1 = MFMA GEMM.  Host-only, no device needed. */
+/* The weights that cmk_iq2_matmul multiplies for IQ2_XXS and these arguments: 0 = exact
+ * (decode shapes), 1 = rounded once to f16 (larger m with in_dim % 8 == 0: the MFMA GEMM,
+ * or the register-dequantising matmul with f16 weights; cmk_iq2_matmul_kernel says
+ * which).  Aligned buffers.  Host-only, no device needed. */
 int cmk_iq2_matmul_path(cmk_dtype x_dtype, size_t m, size_t out_dim, size_t in_dim,
                         cmk_act_quant_mode mode);
+/* Which kernel cmk_iq2_matmul runs for these arguments, aligned buffers and
+ * `workspace_bytes` of workspace (SIZE_MAX: as much as it can use) on 256 CUs:
+ * 0 = the one-row GEMV, the multi-row decode kernel or a portable kernel, 1 = the MFMA
+ * GEMM, 2 = the register-dequantising matmul; a negative cmk_status for arguments that
+ * cmk_iq2_matmul refuses.  For 2 also the rows it takes at a time, the rows of its tiles
+ * (32, 64 or 128; of f32 rows without W8A8 half as many) and the parts of its split over
+ * K; 0 otherwise.  Each pointer may be NULL.  Host-only, no device needed. */
+int cmk_iq2_matmul_kernel(cmk_dtype x_dtype, size_t m, size_t out_dim, size_t in_dim,
+                          cmk_iq2_variant variant, cmk_act_quant_mode mode,
+                          size_t workspace_bytes, size_t *rows_per_pass, int *row_tile,
+                          int *splits);
 
 /* ------------------------------------------------------------------------ */
 /* Thin HIP runtime wrappers for hosts that do not link HIP themselves (the   */
