@@ -43,3 +43,26 @@ def test_refused_arguments(cabi):
         cabi.matmul_kernel(cabi.CMK_F32, 1, 0, 256)
     with pytest.raises(cabi.CmkError, match="workspace too small"):
         cabi.matmul_kernel(cabi.CMK_F32, 512, 14336, 4096, workspace_bytes=0)
+
+
+@pytest.mark.parametrize("x,m,n,k,v,w8a8,kernel", [
+    # staged rows: decode launches are the faster ones at short K
+    ("bf16", 5, 2048, 2048, 1, False, "decode"), ("f32", 8, 4096, 1024, 2, False, "decode"),
+    ("f32", 8, 28672, 1024, 1, False, "decode"), ("bf16", 5, 4096, 4096, 1, False, "register_matmul"),
+    ("bf16", 8, 4096, 1024, 1, True, "register_matmul"), ("bf16", 8, 28672, 1024, 1, True, "decode"),
+    ("bf16", 5, 12288, 2048, 1, False, "register_matmul"), ("bf16", 5, 12288, 1024, 1, False, "decode"),
+    ("f32", 8, 12288, 1024, 2, False, "register_matmul"), ("f32", 5, 20480, 2048, 2, False, "decode"),
+    ("f16", 2, 4099, 1027, 1, False, "decode"), ("f32", 5, 4099, 1027, 1, False, "register_matmul"),
+    ("bf16", 5, 5000, 900, 1, False, "decode"),
+    ("f32", 16, 4096, 512, 1, False, "decode"), ("f32", 16, 4096, 512, 2, False, "register_matmul"),
+    ("f32", 17, 4096, 512, 1, False, "register_matmul"),
+    # two rows of long ones
+    ("f32", 2, 1536, 28672, 3, False, "decode"), ("f32", 2, 2048, 16384, 3, False, "register_matmul"),
+    ("f32", 3, 1536, 28672, 1, False, "register_matmul"),
+    # few f16 rows of many columns
+    ("f16", 2, 28672, 2048, 1, False, "decode"), ("f16", 5, 28672, 2048, 1, False, "register_matmul"),
+    ("f16", 2, 28672, 4096, 1, False, "register_matmul")])
+def test_lines_between_kernels(cabi, x, m, n, k, v, w8a8, kernel):
+    code = {"f32": cabi.CMK_F32, "f16": cabi.CMK_F16, "bf16": cabi.CMK_BF16}[x]
+    mode = cabi.CMK_ACT_QUANT_W8A8 if w8a8 else cabi.CMK_ACT_QUANT_OFF
+    assert cabi.matmul_kernel(code, m, n, k, variant=v, mode=mode)["kernel"] == kernel
