@@ -255,7 +255,7 @@ MmUse mm_use(Path p, int variant, const void* x, int x_dtype, bool w8a8, const u
   if (workspace != nullptr && aligned(workspace, 16))
     u.budget = std::min(workspace_bytes,
                         workspace_for(p, variant, w8a8, x_dtype, d.m, d.out_dim, d.in_dim));
-  u.rows = cmk::iq_mm_rows_per_pass(x_dtype, w8a8, x, d.m, d.out_dim, d.in_dim, workspace,
+  u.rows = cmk::iq_mm_rows_per_pass(x_dtype, w8a8, p == Path::Gemm, x, d.m, d.in_dim, workspace,
                                     u.budget);
   return u;
 }

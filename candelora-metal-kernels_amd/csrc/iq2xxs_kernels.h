@@ -98,9 +98,11 @@ hipError_t launch_split_sum(const float* partials, uint32_t splits, uint64_t n, 
 // copied, bf16 scaled by a power of two, f32 as head / tail row pairs of the scaled row,
 // W8A8 as the integer q.  row_inv (m floats; unused for f16 without W8A8) gets what the
 // rows were multiplied by.  x needs its element's alignment only, rows 16 bytes.
+// block_inv (bf16 and f32 without W8A8; m * ceil(in_dim / 256) floats): super-blocks far below
+// their row are scaled up by themselves (iq_stage.hip); row_inv of such a row is negative.
 hipError_t launch_iq_stage_rows(const void* x, int x_dtype, bool w8a8, uint32_t m,
                                 uint32_t in_dim, uint32_t pitch, float* row_inv, void* rows,
-                                hipStream_t stream);
+                                hipStream_t stream, float* block_inv = nullptr);
 
 // MFMA matmul with exact weights, dequantised in registers (variant 0 .. 3, any m).
 // Needs weight_bytes 16-byte and weight_scales 2-byte aligned and below 2 GB
@@ -121,7 +123,7 @@ size_t iq_mm_scratch_bytes(int x_dtype, bool w8a8, bool f16_weights, const void*
                            uint32_t out_dim, uint32_t in_dim);
 bool iq_mm_scratch_serves(int x_dtype, bool w8a8, bool f16_weights, uint32_t m, uint32_t out_dim,
                           uint32_t in_dim, size_t budget);
-uint32_t iq_mm_rows_per_pass(int x_dtype, bool w8a8, const void* x, uint32_t m, uint32_t out_dim,
+uint32_t iq_mm_rows_per_pass(int x_dtype, bool w8a8, bool f16_weights, const void* x, uint32_t m,
                              uint32_t in_dim, const void* scratch, size_t budget);
 // Tile rows (staged rows for f32 without W8A8) and k splits of a pass of `rows` aligned rows.
 void iq_mm_shape(int x_dtype, bool w8a8, bool f16_weights, uint32_t rows, uint32_t out_dim,
