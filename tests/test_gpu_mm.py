@@ -1,7 +1,7 @@
-"""The register-dequantising MFMA matmul at the edges of its tiles: row tiles of 32, 64 and
-128, column tiles of 64 to 256, one and several super-blocks (the parts of K that waves share
-run out unevenly), partial and odd K, staged rows of every type, W8A8, and less scratch than
-it would like.
+"""The register-dequantising MFMA matmul at the edges of its 32-row tiles (test_gpu_mm_tiles.py
+has the wider ones): one and several super-blocks (the parts of K that waves share run out
+unevenly), partial and odd K, staged rows of every type, W8A8, and less scratch than it would
+like.  The smallest shapes stay on the decode launches, in IQ2_XXS more of them.
 
 Bar: exact weights and fp32 sums, so the bars of the decode kernels hold: cond <= 1e-5 and
 rel <= 1e-3 against the fp64 oracle (test_gpu_parity.py).  IQ2_XXS above 16 rows (W8A8 32)
@@ -51,6 +51,8 @@ def _run(pkg, v, x, n, k, wb, ws, w8a8):
     (128, 256, 768, "f16", False), (129, 100, 4104, "f16", False), (300, 70, 512, "f16", False),
     (20, 96, 2051, "f16", False), (40, 333, 777, "bf16", False), (16, 64, 4096, "bf16", False),
     (65, 130, 1000, "f32", False), (12, 33, 2872, "f32", False), (17, 40, 515, "f32", False),
+    (20, 600, 2051, "f16", False), (16, 300, 4096, "bf16", False), (12, 400, 2872, "f32", False),
+    (17, 2050, 515, "f32", False),
     (33, 96, 1024, "f16", True), (70, 65, 1291, "bf16", True), (130, 64, 2304, "f32", True)])
 def test_tile_edges(pkg, oracle, inputs, dev, v, m, n, k, dtype, w8a8):  # noqa: F811
     wb, ws = random_weights(oracle, v, n, k, seed=m + 3 * n + k)
