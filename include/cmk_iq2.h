@@ -116,10 +116,12 @@ typedef enum cmk_act_quant_mode {
  * into parts, one workgroup each, whose sums meet in the workspace and are
  * added in part order by the part that finishes last (the same results on
  * every run, equal to the unsplit launch up to fp32 rounding).  The
- * register-dequantising matmul (exact weights up to 16 rows and in the formats
- * other than IQ2_XXS) stages f32, bf16, W8A8 and unaligned rows in the workspace
- * and splits K as far as it has room; with less than the query reports it takes
- * the rows in passes, and with too little for 128 rows the decode kernel runs.
+ * register-dequantising matmul (weights as cmk_iq2_matmul_path says for IQ2_XXS,
+ * exact in the other formats) stages f32, bf16, W8A8 and unaligned rows in the
+ * workspace, at most 256 MB of them at a time, and splits K as far as it has room;
+ * with less than the query reports it takes fewer rows at a time and splits less
+ * (the same products, summed in another order), and with too little for 128 rows
+ * or for those there are the kernels that need none run.
  * The workspace needs no initial contents; launches that share one must be ordered (one
  * stream).
  */
@@ -135,11 +137,14 @@ int cmk_iq2_matmul(const void *x, cmk_dtype x_dtype, size_t x_len, size_t m,
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * hosts that forbid allocation).  No counterpart in the reference, whose
  * dispatch allocates its output per call (src/iq2_matmul.rs:261).  Same
- * arguments, checks, kernels and results as cmk_iq2_matmul; the scratch the
- * launch needs (the MFMA GEMM's staged rows, row scales and k-split partials)
- * comes from an array inside the library, one per device, of
- * CMK_IQ2_NOALLOC_SCRATCH_BYTES bytes.  Arguments that need more fail with
- * CMK_ERR_INVALID_ARGUMENT before anything is launched.  The call performs no
+ * arguments, checks, kernels and results as cmk_iq2_matmul with a workspace of
+ * CMK_IQ2_NOALLOC_SCRATCH_BYTES bytes, an array inside the library, one per
+ * device.  Calls of two rows and more use it, in every format and from the
+ * smallest batches on: staged rows and their scales, partial sums of a split of K,
+ * and the multi-row kernel's arrival words.  Arguments for which cmk_iq2_matmul
+ * would refuse a workspace of that size fail with CMK_ERR_INVALID_ARGUMENT before
+ * anything is launched; the register-dequantising matmul, which takes what there
+ * is, runs in more passes, or with less of a split, instead.  The call performs no
  * device allocation: the array is part of the code object and lives until the
  * process ends; the first call on a device looks up its address once.  All
  * calls on one device share that device's array and nothing clears it between
@@ -157,7 +162,9 @@ int cmk_iq2_matmul_noalloc(const void *x, cmk_dtype x_dtype, size_t x_len, size_
  * launch never allocates; callers that get a non-zero size pass a buffer of at
  * least that many bytes.  Same argument validation as cmk_iq2_matmul.  The
  * size includes the multi-row kernel's optional split over K, counted for
- * 256 CUs (a device with fewer CUs never splits more). */
+ * 256 CUs (a device with fewer CUs never splits more), or what the
+ * register-dequantising matmul would best have; with less, or none, those calls
+ * run too, if more slowly. */
 int cmk_iq2_matmul_workspace_size(cmk_dtype x_dtype, size_t m, size_t out_dim, size_t in_dim,
                                   cmk_iq2_variant variant, cmk_act_quant_mode mode,
                                   size_t *bytes);
