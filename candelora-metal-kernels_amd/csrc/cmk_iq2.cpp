@@ -44,17 +44,13 @@ int hip_fail(hipError_t e, const char* what) {
 size_t bytes_per_block(int v) { return v == CMK_IQ2_XXS ? 64 : cmk::variant_bytes_per_block(v); }
 size_t scales_per_block(int v) { return v == CMK_IQ2_XXS ? 2 : cmk::variant_scales_per_block(v); }
 
-// Largest m served by the GEMV family (above it: the MFMA GEMM).  The GEMV
-// multiplies exact weights (the GEMM rounds them to f16) and takes up to 16
-// rows in one launch, which at 9-16 rows is also faster than the GEMM for
-// f16 / bf16 x at the decode shapes (K=4096: 18.9-19.9 against 23.1-27.9 us at
-// N=14336; K=8192, N=28672: 54 against 86 us), the one exception measured being
-// N=4096 (16.1 against 13.2 us at 16 rows).
+// Largest m of IQ2_XXS whose weights are exact; above it they are rounded to f16
+// (with in_dim % 8 == 0 and aligned buffers).  Which kernel serves either side is
+// decided by iq_mm_pays; where it is not the matmul in registers, up to these rows
+// go in one launch of the multi-row decode kernel (16, of int8 W8A8 rows 32), more
+// on the MFMA GEMM.
 constexpr size_t kGemvMaxM = 16;
 constexpr size_t kGemvMaxMF32 = 16;
-// W8A8 activations are int8 on the multi-row kernel, 32 rows per launch: at
-// 24 to 32 rows it is level in time with the GEMM (which rounds the weights
-// to f16) and its sums are exact.
 constexpr size_t kGemvMaxMW8A8 = 32;
 constexpr size_t kWorkspaceAlign = 256;
 
@@ -435,8 +431,8 @@ int cmk_iq2_matmul(const void* x, cmk_dtype x_dtype, size_t x_len, size_t m,
   float* partials =
       need_ws > head_ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + head_ws)
                         : nullptr;
-  // IQ2_XS / IQ2_S / IQ3_S with aligned weights: the multi-row decode kernel
-  // (W8A8 scales computed there; the workspace stays unused)
+  // IQ2_XS / IQ2_S / IQ3_S with aligned weights where the matmul in registers does not
+  // run: the multi-row decode kernel (W8A8 scales computed there)
   const bool variant_rows = p == Path::Variant && aligned(weight_bytes, 16) &&
                             aligned(weight_scales, 2) &&
                             cmk::variant_rows_supported((int)variant, dims.out_dim, dims.in_dim,

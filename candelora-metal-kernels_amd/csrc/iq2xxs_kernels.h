@@ -10,8 +10,8 @@ namespace cmk {
 // dtype / output kind codes shared with the ABI: 0 = f32, 1 = f16, 2 = bf16.
 
 // Dense dequantisation, out[out_dim, in_dim], of variant 0 (IQ2_XXS), 1 (IQ2_XS),
-// 2 (IQ2_S) or 3 (IQ3_S).  Any alignment of the weight buffers; out aligned to its
-// element.
+// 2 (IQ2_S) or 3 (IQ3_S).  IQ2_XXS: weight_bytes 8-byte, weight_scales 2-byte aligned;
+// the others: any alignment.  out aligned to its element.
 hipError_t launch_iq_dequant(int variant, const uint8_t* wb, const uint8_t* ws, void* out,
                              int out_kind, uint32_t out_dim, uint32_t in_dim, int num_cus,
                              hipStream_t stream);

@@ -84,12 +84,8 @@ __device__ __forceinline__ void decode_group(const uint8_t* __restrict__ wb,
   uint32_t sgn;
   float dl;
   if constexpr (V == 0) {
-    uint32_t aux_s;
-    if constexpr (kAligned) {
-      aux_s = *reinterpret_cast<const uint32_t*>(q + 8 * sb + 4);
-    } else {
-      aux_s = dequant_u16<false>(q + 8 * sb + 4) | (dequant_u16<false>(q + 8 * sb + 6) << 16);
-    }
+    static_assert(kAligned, "IQ2_XXS buffers are aligned");
+    const uint32_t aux_s = *reinterpret_cast<const uint32_t*>(q + 8 * sb + 4);
     mag = grid[q[8 * sb + w]];
     sgn = dequant_ksigns((aux_s >> (7 * w)) & 0x7Fu);
     dl = (d * (0.5f + (float)(aux_s >> 28))) * 0.25f;
@@ -279,7 +275,10 @@ static hipError_t launch_dequant_v(const uint8_t* wb, const uint8_t* ws, void* o
                                    hipStream_t stream) {
   if (reinterpret_cast<uintptr_t>(wb) % 8 == 0 && reinterpret_cast<uintptr_t>(ws) % 2 == 0)
     return launch_dequant_kind<V, true>(wb, ws, out, out_kind, out_dim, in_dim, num_cus, stream);
-  return launch_dequant_kind<V, false>(wb, ws, out, out_kind, out_dim, in_dim, num_cus, stream);
+  if constexpr (V == 0)  // (cmk_iq2_dequantize refuses unaligned IQ2_XXS buffers)
+    return hipErrorInvalidValue;
+  else
+    return launch_dequant_kind<V, false>(wb, ws, out, out_kind, out_dim, in_dim, num_cus, stream);
 }
 
 hipError_t launch_iq_dequant(int variant, const uint8_t* wb, const uint8_t* ws, void* out,
